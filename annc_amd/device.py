@@ -244,10 +244,14 @@ def unique_gather(table: torch.Tensor, keys: torch.Tensor, col: int = 0, stream=
     uniq = torch.empty(max(n, 1), dtype=torch.int64, device=table.device)
     idx = torch.empty(n, dtype=torch.int32, device=table.device)
     out = torch.empty((max(n, 1), dim), dtype=torch.float32, device=table.device)
-    check(_lib.lib().annc_hip_unique_gather(stream_ptr(stream), ptr(table.contiguous()), rows, dim,
-                                            ptr(k2) + 8 * col if n else None, k2.stride(0), n,
-                                            ptr(nu), ptr(uniq), ptr(idx), ptr(out)))
-    (stream if stream is not None else torch.cuda.current_stream()).synchronize()
+    rc = _lib.lib().annc_hip_unique_gather(stream_ptr(stream), ptr(table.contiguous()), rows, dim,
+                                           ptr(k2) + 8 * col if n else None, k2.stride(0), n,
+                                           ptr(nu), ptr(uniq), ptr(idx), ptr(out))
+    if rc != _lib.INVALID_ARGUMENT:  # (refused before any launch)
+        # also after a failure: a kernel already queued writes the count, and
+        # pinned memory that is given back is handed out again at once
+        (stream if stream is not None else torch.cuda.current_stream()).synchronize()
+    check(rc)
     u = int(nu.item())
     return uniq[:u], idx, out[:u]
 

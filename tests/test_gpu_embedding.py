@@ -943,3 +943,30 @@ def test_reduce_mean_custom_call(m, n, where):
         assert np.isnan(out).all()
     else:
         np.testing.assert_allclose(out, want, rtol=1e-5 + 2e-7 * np.sqrt(m))
+
+
+def test_unique_gather_waits_before_it_reports_a_failure(monkeypatch):
+    """The count is in pinned host memory: a call that fails after its kernels
+    are queued gives that memory back only once they have run."""
+    note("unique_gather failing after its launches")
+    d = device()
+    lib = dev._lib.lib()
+
+    class FailsAfterLaunch:
+        def annc_hip_unique_gather(self, *args):
+            assert lib.annc_hip_unique_gather(*args) == dev._lib.OK
+            return dev._lib.INTERNAL
+
+        def __getattr__(self, name):
+            return getattr(lib, name)
+
+    table = torch.randn(1000, 16, device=d)
+    keys = torch.arange(1000, device=d)
+    x = torch.randn(4096, 4096, device=d)
+    torch.cuda.synchronize()
+    monkeypatch.setattr(dev._lib, "lib", FailsAfterLaunch)
+    for _ in range(20):  # a few ms of work ahead of the launches
+        x @ x
+    with pytest.raises(dev._lib.AnncError):
+        dev.unique_gather(table, keys)
+    assert torch.cuda.current_stream().query()
