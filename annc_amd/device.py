@@ -370,11 +370,14 @@ def hashed_embedding_bags(tables: Sequence[torch.Tensor], num_buckets: Sequence[
 
 
 def _int64s(values: Sequence[int]) -> array:
-    """A host int64 array of the values (a third of numpy's time for a list)."""
+    """A host int64 array of the values (a third of numpy's time for a list of
+    ints; anything else, as rows of one value or floats, goes through numpy)."""
+    if not isinstance(values, (list, tuple)):
+        values = list(values)
     try:
         return array("q", values)
-    except TypeError:  # floats
-        return array("q", np.asarray(list(values), dtype=np.int64).tolist())
+    except TypeError:
+        return array("q", np.asarray(values, dtype=np.int64).ravel().tolist())
 
 
 def _address(values: array) -> int:

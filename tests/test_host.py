@@ -8,6 +8,7 @@ import re
 
 import numpy as np
 import pytest
+import torch
 
 from annc_amd import _lib, flags, tf_ops, xla
 from annc_amd._lib import AnncError
@@ -308,3 +309,13 @@ def test_batch_matmul_add_sigmoid_error_messages(case):
         tf_ops.kp_fused_batch_matmul_add_sigmoid(mk(case["lhs_shape"]), mk(case["rhs_shape"]),
                                                  mk(case["bias_shape"]))
     assert case["message"] in e.value.message
+
+
+@pytest.mark.parametrize("values", [[3, 5, 7], (3, 5, 7), np.array([3, 5, 7], np.int32),
+                                    np.array([[3], [5], [7]]), [3.0, 5.9, 7.2], [np.int64(3), 5, True + 6],
+                                    range(3, 8, 2), (v for v in (3.0, 5.0, 7.0)), bytes([3, 5, 7]),
+                                    torch.tensor([3, 5, 7])], ids=str)
+def test_host_int64_arrays_of_any_sequence(values):
+    """Bucket counts and slice bounds reach the library as int64 whatever holds
+    them: lists, arrays of any shape and type, generators."""
+    assert list(dev._int64s(values)) == [3, 5, 7]
