@@ -64,18 +64,10 @@ class MLPTower:
 
     With `fuse_score` (the default) a tower whose last layer has one output
     runs its last two layers as one kernel (annc_hip_dense_score) when the
-    shapes allow and the batch has `fuse_min_rows` to FUSE_MAX_ROWS rows: the
-    scoring dot reads the hidden layer from registers, and that hidden layer
-    reaches memory only with `keep_hidden`.  Every other layer, and the tail
-    when it does not fit, is one GEMM launch.  The fused kernel gives each 16
-    rows a workgroup that streams the whole hidden-layer weight, so a round of
-    256 workgroups takes as long for 2304 rows as for 4096, and each further
-    round as long again, while the GEMM's tiles follow the batch.  Steps of a
-    1024-512-256-1 tower, fused / unfused, us: 1024 rows 25.7 / 25.6, 2048
-    31.9 / 30.7, 2304 36.3 / 38.4, 4096 42.7 / 44.7, 6144 64.4 / 62.4, 8192
-    72.4 / 72.0, 16384 132.6 / 122.6."""
-
-    FUSE_MAX_ROWS = 5120
+    shapes allow, the batch has at least `fuse_min_rows` rows and fuses_at()
+    finds it faster: the scoring dot reads the hidden layer from registers, and
+    that hidden layer reaches memory only with `keep_hidden`.  Every other
+    layer, and the tail when it does not fit, is one GEMM launch."""
 
     def __init__(self, weights: Sequence[np.ndarray], biases: Sequence[np.ndarray],
                  device: torch.device | str = "cuda", packed: bool = True,
@@ -97,6 +89,24 @@ class MLPTower:
         if fuse_score and packed and len(self.layers) >= 2:
             hid, last = self.layers[-2].weight, self.layers[-1].weight
             self.fused_tail = last.n == 1 and dev.dense_score_fits(hid.k, hid.n)
+
+    def fuses_at(self, rows: int) -> bool:
+        """Whether a batch of `rows` runs the tail as one kernel.
+
+        That kernel gives each 16 rows a workgroup that streams the whole
+        hidden-layer weight: up to 4096 rows are one round of workgroups, and
+        each further round streams the weight again, while the GEMM's tiles
+        follow the batch.  Steps of towers with a tail of K -> N -> 1, fused /
+        unfused, us: 512 -> 256 at 4096 rows 45.0 / 48.2, 4112 63.9 / 62.1, 5120
+        64.5 / 62.6, 8192 75.2 / 74.5, 16384 134 / 127; 1024 -> 256 4112 104 / 94,
+        16384 259 / 234; 1024 -> 128 5120 65.1 / 62.2; smaller weights 256 -> 128
+        5120 26.7 / 29.9, 16384 45.6 / 49.1; 512 -> 128 5120 42.1 / 44.4, 16384
+        72.9 / 73.0, 32768 137 / 131; 512 -> 64 32768 119 / 122; 256 -> 256 16384
+        55.4 / 56.9, 32768 97 / 86."""
+        if not self.fused_tail or rows < self.fuse_min_rows:
+            return False
+        hid = self.layers[-2].weight
+        return rows <= 4096 or (hid.k * hid.n < 1 << 17 and rows * hid.k * hid.n <= 1 << 30)
 
     @property
     def widths(self) -> list[int]:
@@ -142,7 +152,7 @@ class MLPTower:
         """x: [batch, k0] (any row stride).  Returns the final [batch, 1] buffer."""
         bufs = self.buffers(x.shape[0])
         h = x
-        fused = self.fused_tail and self.fuse_min_rows <= x.shape[0] <= self.FUSE_MAX_ROWS
+        fused = self.fuses_at(x.shape[0])
         plain = len(self.layers) - (2 if fused else 0)
         for layer, out in zip(self.layers[:plain], bufs):
             dev.gemm(h, layer.weight, bias=layer.bias, epilogue=layer.activation, out=out,

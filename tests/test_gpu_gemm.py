@@ -296,6 +296,27 @@ def test_tower_fuses_its_tail_above_2048_rows(batch):
         assert np.isfinite(hidden).all()
 
 
+@pytest.mark.parametrize("widths,batch,fused", [
+    ((64, 512, 256, 1), 4096, True), ((64, 512, 256, 1), 4097, False),
+    ((64, 256, 128, 1), 4097, True), ((64, 256, 128, 1), 32768, True),
+    ((64, 256, 128, 1), 32769, False), ((64, 512, 128, 1), 16385, False)])
+def test_tower_tail_past_one_round_of_rows(widths, batch, fused):
+    """Past 4096 rows the tail stays one kernel where its weight is small and
+    the batch is not too large for it, else it is two GEMM launches (which write
+    the hidden layer's buffer)."""
+    note(f"tower {widths} tail path at batch {batch}")
+    g = workloads.rng(batch)
+    ws = [workloads.glorot_uniform(g, a, b) for a, b in zip(widths, widths[1:])]
+    bs = [(g.standard_normal(b) * 0.01).astype(np.float32) for b in widths[1:]]
+    x = g.standard_normal((batch, widths[0])).astype(np.float32)
+    tower = MLPTower(ws, bs, device=device())
+    bufs = tower.buffers(batch)
+    bufs[-2].fill_(float("nan"))
+    y = to_host(tower(to_dev(x)))
+    np.testing.assert_allclose(y, ora.mlp_tower(x, ws, bs), rtol=1e-3, atol=1e-5)
+    assert np.isnan(to_host(bufs[-2])).all() == fused
+
+
 @pytest.mark.parametrize("widths,offset", [((512, 256, 1), 1), ((512, 256, 1), 4), ((512, 96, 1), 0)])
 def test_tower_tail_fallbacks(widths, offset):
     """Towers whose tail the fused kernel does not take run it as two GEMM
