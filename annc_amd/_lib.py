@@ -70,6 +70,7 @@ _PROTOTYPES = {
     "annc_layout_matmul_pack_rhs": (_i32, [_i64, _i64, _c_void_p, _c_void_p]),
     "annc_layout_matmul_unpack_rhs": (_i32, [_i64, _i64, _c_void_p, _c_void_p]),
     "annc_hip_layout_matmul_pack_rhs": (_i32, [_c_void_p, _i64, _i64, _c_void_p, _c_void_p]),
+    "annc_hip_gemm_tile": (_i32, [_i64] * 4),
     "annc_hip_gemm": (_i32, [_c_void_p, _i64, _i64, _i64, _i64,
                              _c_void_p, _i64, _i64,
                              _c_void_p, _i64, _i64, _i32,

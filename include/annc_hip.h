@@ -219,6 +219,15 @@ int annc_hip_gemm(void* stream, int64_t batch, int64_t m, int64_t n, int64_t k,
                   const float* bias, int epilogue,
                   float* c, int64_t ldc, int64_t stride_c);
 
+/* The tile in which annc_hip_gemm runs a product (nothing is launched): 0 to 4,
+ * 256x128, 128x128, 128x64, 64x64 or 64x32 with fp32 operands as three bf16
+ * pieces; 5 to 7, 64x64, 64x32 or 128x64 on the fp32 matrix instruction; 8
+ * more where the N % 32 tail columns take a second launch; -1 where another
+ * kernel runs (N <= 4, at most 256 32x32 blocks, bad sizes).  Row strides of
+ * 2^25 floats (A) or 2^27 (row-major B) and more, and ANNC_GEMM_PIPE, are not
+ * looked at. */
+int annc_hip_gemm_tile(int64_t batch, int64_t m, int64_t n, int64_t k);
+
 /* Tower tail in one kernel: the last hidden layer on a packed weight and the
  * N -> 1 scoring layer after it,
  *   h      = epi( A . B + bias )                       [m, n]
