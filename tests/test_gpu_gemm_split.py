@@ -125,7 +125,9 @@ TINY_CASES = [(1, 1, 512, 1024), (1, 17, 33, 64), (1, 16, 47, 545), (1, 15, 8, 2
               # 32x32 blocks (the small kernel): edges, K tails and K < 32, fewer k-blocks
               # than waves and more than its ring of 8 x 4, K split over workgroups
               (1, 257, 1000, 1024), (1, 500, 500, 31), (1, 290, 260, 65), (1, 300, 300, 1311),
-              (3, 100, 480, 100), (1, 8190, 17, 320), (1, 128, 1000, 3100)]
+              (3, 100, 480, 100), (1, 8190, 17, 320), (1, 128, 1000, 3100),
+              # from K = 2048 up to 128 blocks (and not at 2047, nor past them)
+              (1, 217, 448, 2048), (1, 217, 448, 2047), (4, 33, 500, 2081), (1, 300, 448, 2048)]
 
 
 @pytest.mark.parametrize("batch,m,n,k", TINY_CASES)
