@@ -4,6 +4,7 @@ smaller ones have to come out as the fp32 instruction gives them."""
 import pytest
 import torch
 
+from annc_amd import _lib
 from annc_amd import device as dev
 from tests.gpu_util import device, note
 
@@ -62,15 +63,16 @@ PLANTS = [_denormal_row, _denormal_column, _zero_pieces, _hidden_in_an_ordinary_
           _large_a_small_b, _small_by_ordinary]
 
 
-# one shape of each tile, whole and ragged in K and N, one batched
-@pytest.mark.parametrize("batch,m,n,k", [(1, 16384, 512, 1056), (1, 8195, 1000, 1023),
-                                         (1, 4096, 1024, 1024), (1, 3000, 544, 1055),
-                                         (1, 2047, 301, 845), (1, 4100, 96, 1000),
-                                         (1, 1025, 512, 1024), (6, 700, 520, 577)])
+# each split tile (256x128 ... 64x32), whole and ragged in K and N, two batched
+@pytest.mark.parametrize("batch,m,n,k,tile", [
+    (1, 16384, 512, 1056, 0), (1, 4096, 1024, 1024, 1), (1, 8195, 1000, 1023, 2),
+    (1, 3000, 544, 1055, 2), (1, 2047, 301, 845, 3), (1, 1025, 512, 1024, 3),
+    (1, 4100, 96, 1000, 4), (3, 451, 704, 192, 2), (3, 512, 612, 577, 3)])
 @pytest.mark.parametrize("plant", PLANTS)
-def test_small_and_large_operands(plant, batch, m, n, k):
+def test_small_and_large_operands(plant, batch, m, n, k, tile):
     note(f"GEMM operand range {plant.__name__} {batch}x{m}x{n}x{k}")
     device()
+    assert _lib.lib().annc_hip_gemm_tile(batch, m, n, k) == tile
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
     shape = (m, k) if batch == 1 else (batch, m, k)
     a = torch.randn(shape, generator=g, device="cuda").relu_()

@@ -1,21 +1,47 @@
-"""The split-operand GEMM (gemm_split.h: fp32 operands as three bf16 pieces)
-and the choice between its tiles and the short-K fp32 kernel."""
-import numpy as np
+"""The split-operand GEMM (gemm_split.h: fp32 operands as three bf16 pieces),
+the fp32 pipeline beside it, the choice between their tiles, and the kernels
+for few blocks."""
 import pytest
 import torch
 
-from annc_amd import EPI_RELU
+from annc_amd import EPI_RELU, _lib
 from annc_amd import device as dev
 from tests.gpu_util import device, note
 
 pytestmark = pytest.mark.gpu
 
-# sizes one past or short of a tile, a 32-column panel, a k-block and a stage;
-# together they reach every tile, with whole and partial last panels
-CASES = [(1, 8195, 1024, 545), (1, 8193, 1001, 577), (1, 4099, 992, 865), (1, 2049, 1000, 1024),
-         (1, 4097, 512, 1023), (1, 2050, 301, 845), (1, 2047, 512, 1055), (1, 1023, 512, 1024),
-         (1, 16390, 16, 1023), (1, 8200, 96, 97), (1, 3000, 70, 33), (1, 4096, 96, 20),
-         (1, 1025, 1024, 256), (1, 4096, 64, 512), (5, 300, 288, 577), (3, 65, 2080, 129)]
+# (batch, m, n, k) and the tile that runs it: 0-4 split 256x128, 128x128, 128x64,
+# 64x64, 64x32; 5-7 fp32 64x64, 64x32, 128x64; + 8: the tail columns in a second
+# launch.  Sizes one past or short of a tile, a 32-column panel, a k-block and a
+# stage: every tile with whole and ragged K and N, one product and batches
+# (128x128 takes whole panels only).  The first sixteen have longer K.
+CASES = [
+    (1, 8195, 1024, 545, 2), (1, 8193, 1001, 577, 2), (1, 4099, 992, 865, 0),
+    (1, 2049, 1000, 1024, 9), (1, 4097, 512, 1023, 1), (1, 2050, 301, 845, 3),
+    (1, 2047, 512, 1055, 3), (1, 1023, 512, 1024, 4), (1, 16390, 16, 1023, 6),
+    (1, 8200, 96, 97, 6), (1, 3000, 70, 33, 6), (1, 4096, 96, 20, 6), (1, 1025, 1024, 256, 2),
+    (5, 300, 288, 577, 6), (3, 65, 2080, 129, 5), (1, 4100, 96, 1000, 4),
+    (1, 2689, 1536, 32, 0), (1, 16385, 197, 64, 0), (1, 3327, 1280, 33, 0), (1, 14080, 257, 33, 0),
+    (7, 897, 640, 32, 0), (3, 3587, 321, 64, 0), (5, 515, 1536, 33, 0), (7, 1923, 261, 33, 0),
+    (1, 4099, 640, 128, 1), (1, 6147, 512, 33, 1), (3, 707, 1152, 128, 1), (7, 257, 1408, 33, 1),
+    (1, 769, 1280, 192, 2), (1, 3587, 257, 192, 2), (1, 2179, 704, 97, 2), (1, 1539, 645, 161, 2),
+    (3, 451, 704, 192, 2), (7, 193, 577, 192, 2), (5, 259, 1024, 97, 2), (7, 65, 1157, 165, 2),
+    (1, 705, 704, 384, 3), (1, 513, 897, 256, 3), (1, 1345, 384, 225, 3), (1, 2691, 165, 193, 3),
+    (7, 65, 640, 512, 3), (3, 67, 1428, 256, 3), (3, 65, 1408, 357, 3), (3, 131, 916, 225, 3),
+    (1, 385, 640, 640, 4), (1, 1153, 193, 128, 4), (1, 323, 768, 353, 4), (1, 1153, 193, 101, 4),
+    (2, 384, 352, 768, 4), (2, 579, 193, 128, 4), (3, 385, 197, 97, 4),
+    (1, 515, 1024, 32, 5), (1, 4097, 101, 32, 5), (1, 323, 1536, 33, 5), (1, 8963, 33, 33, 5),
+    (5, 65, 896, 32, 5), (3, 131, 901, 32, 5), (2, 129, 1408, 33, 5), (7, 65, 660, 37, 5),
+    (1, 897, 288, 32, 6), (1, 2049, 97, 32, 6), (1, 195, 1280, 33, 6), (1, 3073, 65, 33, 6),
+    (2, 451, 288, 32, 6), (3, 1535, 33, 32, 6), (5, 195, 256, 33, 6), (5, 963, 33, 37, 6),
+    (1, 2943, 896, 32, 7), (1, 11007, 129, 32, 7), (1, 11521, 288, 33, 7), (1, 12547, 212, 33, 7),
+    (3, 707, 1152, 32, 7), (7, 2816, 69, 32, 7), (5, 3583, 192, 33, 7), (7, 1791, 193, 37, 7),
+    (1, 6657, 1183, 33, 8), (5, 640, 1281, 33, 9), (1, 2819, 709, 97, 10), (7, 65, 1172, 709, 11),
+    (1, 1089, 468, 896, 12), (5, 257, 1285, 33, 13), (3, 129, 927, 325, 14), (1, 2563, 1537, 32, 15)]
+
+
+def _tile(batch, m, n, k):
+    return _lib.lib().annc_hip_gemm_tile(batch, m, n, k)
 
 
 def _operands(batch, m, n, k, lda_pad, seed):
@@ -26,45 +52,72 @@ def _operands(batch, m, n, k, lda_pad, seed):
     return a, b
 
 
-def _check(got, a, b, bias):
-    """|error| <= 2 * (K/16 + 32) * 2^-24 * |A||B|: the large products round
-    once per 16 k (by up to one unit, as the matrix units truncate), their
-    corrections are 2^-8 of them, and at most 32 roundings more (pieces left
-    out, groups added, bias)."""
+def _check(got, a, b, bias, tile):
+    """|error| <= 2 * R * 2^-24 * |A||B|.  Split tiles: R = K/16 + 32, the large
+    products round once per 16 k (by up to one unit, as the matrix units
+    truncate), their corrections are 2^-8 of them, and at most 32 roundings
+    more (pieces left out, groups added, bias).  The fp32 instruction rounds
+    once per k pair (per k in the tail columns' kernel): R = K/2 + 32 (K + 32)."""
     ref = a.double() @ b.double() + bias.double()
     k = a.shape[-1]
-    bound = 2 * (k / 16 + 32) * 2.0 ** -24 * (a.double().abs() @ b.double().abs() + bias.abs())
-    # (short K runs the fp32 instruction: one rounding per k pair, K <= 512)
-    if k <= 512:
-        bound = bound * (1 + k / 2 / (k / 16 + 32))
+    roundings = 32 + (k if tile >= 8 else k / 16 if tile < 5 else k / 2)
+    bound = 2 * roundings * 2.0 ** -24 * (a.double().abs() @ b.double().abs() + bias.abs())
     err = (got.double() - ref.relu()).abs() - bound
     assert err.max().item() <= 0, f"{(err > 0).sum().item()} out of bounds, worst {err.max().item()}"
 
 
-@pytest.mark.parametrize("batch,m,n,k", CASES)
+@pytest.mark.parametrize("batch,m,n,k,tile", CASES)
 @pytest.mark.parametrize("lda_pad,ldb_pad", [(0, 0), (3, 1)])
-def test_split_gemm_edges(batch, m, n, k, lda_pad, ldb_pad):
+def test_split_gemm_edges(batch, m, n, k, tile, lda_pad, ldb_pad):
     """Every tile at its edges, rows of any alignment, within the bound of the
     64-bit product; packed and row-major B give the same bits."""
     note(f"split GEMM {batch}x{m}x{n}x{k} lda+{lda_pad} ldb+{ldb_pad}")
     device()
+    assert _tile(batch, m, n, k) == tile, "the case has left its tile: take another size"
     a, b = _operands(batch, m, n, k, lda_pad, m + n + k)
     bias = torch.randn(n, device="cuda")
     wide = torch.zeros(b.shape[:-1] + (n + ldb_pad,), device="cuda")
     wide[..., :n] = b
     got = dev.gemm(a, wide[..., :n], bias=bias, epilogue=EPI_RELU)
-    _check(got, a, b, bias)
+    _check(got, a, b, bias, tile)
     if batch == 1:
         packed = dev.gemm(a, dev.pack_weight(b), bias=bias, epilogue=EPI_RELU)
         assert torch.equal(got, packed)
 
 
-@pytest.mark.parametrize("m,n,k", [(1025, 512, 1024), (4096, 512, 1000), (8192, 1000, 640)])
-def test_split_gemm_values_its_pieces_cannot_hold(m, n, k):
-    """Infinite, NaN, largest and smallest operands: what the products of the
-    pieces cannot represent is recomputed with the fp32 instruction."""
-    note(f"split GEMM special values {m}x{n}x{k}")
+# one of each split tile, ragged
+@pytest.mark.parametrize("m,n,k,tile", [(4099, 992, 865, 0), (4097, 512, 1023, 1), (8193, 1001, 577, 2),
+                                        (2050, 301, 845, 3), (1153, 193, 101, 4)])
+def test_one_product_an_output(m, n, k, tile):
+    """Rows of A with one nonzero: of the nine products of the pieces, m*l, l*m
+    and l*l are left out, up to 2^-24 of the operands' product together, and
+    the sum of the others is rounded once: within 2^-23 (the fp32 instruction:
+    2^-24)."""
+    note(f"split GEMM of one nonzero a row {m}x{n}x{k}")
     device()
+    assert _tile(1, m, n, k) == tile
+    g = torch.Generator(device="cuda").manual_seed(m)
+    a = torch.zeros((m, k), device="cuda")
+    a[torch.arange(m, device="cuda"), torch.randint(k, (m,), generator=g, device="cuda")] = \
+        torch.rand(m, generator=g, device="cuda") + 1
+    b = torch.rand((k, n), generator=g, device="cuda") + 1
+    ref = a.double() @ b.double()
+    for w in (b, dev.pack_weight(b)):
+        assert ((dev.gemm(a, w).double() - ref).abs() <= 2.0 ** -23 * ref).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(1025, 512, 1024), (4096, 512, 1000), (8192, 1000, 640),
+                                   (2050, 301, 845), (385, 640, 640), (4097, 512, 1023)])
+@pytest.mark.parametrize("layout", ["row-major", "packed", "batched"])
+def test_split_gemm_values_its_pieces_cannot_hold(m, n, k, layout):
+    """Infinite, NaN, largest and smallest operands: what the products of the
+    pieces cannot represent is recomputed with the fp32 instruction, on packed
+    and row-major B with and without tails, and in every batch."""
+    note(f"split GEMM special values {m}x{n}x{k} {layout}")
+    device()
+    batch = 3 if layout == "batched" else 1
+    tile = _tile(batch, m, n, k)
+    assert tile < 5
     a, b = _operands(1, m, n, k, 0, 7)
     b[:, 5] = b[:, 5].abs() + 0.01
     big = torch.finfo(torch.float32).max
@@ -81,7 +134,14 @@ def test_split_gemm_values_its_pieces_cannot_hold(m, n, k):
     a[201, 9] = 2.0 ** -121
     a[202, 9] = 2.0 ** -140
     zero = torch.zeros(n, device="cuda")
-    got = dev.gemm(a, b)
+    if layout == "batched":  # the values in the middle one
+        a3, b3 = torch.ones((3, m, k), device="cuda"), torch.ones((3, k, n), device="cuda")
+        a3[1], b3[1] = a, b
+        got = dev.gemm(a3, b3)
+        assert (got[0] == k).all() and (got[2] == k).all()
+        got = got[1]
+    else:
+        got = dev.gemm(a, dev.pack_weight(b) if layout == "packed" else b)
     ref = a.double() @ b.double()
     for r in (3, 70, 130, 200):
         # (a sum of -inf and inf terms is NaN in both)
@@ -98,7 +158,7 @@ def test_split_gemm_values_its_pieces_cannot_hold(m, n, k):
         assert ((x - y).abs() <= bound).all(), r
     ok = torch.ones(m, dtype=torch.bool, device="cuda")
     ok[[3, 70, 130, 200, 201, 202]] = False
-    _check(got[ok][:, keep].relu(), a[ok], b[:, keep], zero[keep])
+    _check(got[ok][:, keep].relu(), a[ok], b[:, keep], zero[keep], tile)
 
 
 def test_row_stride_past_32_bit_offsets():
@@ -114,7 +174,7 @@ def test_row_stride_past_32_bit_offsets():
         a.copy_(src)
         bias = torch.randn(n, device="cuda")
         for w in (b, dev.pack_weight(b)):
-            _check(dev.gemm(a, w, bias=bias, epilogue=EPI_RELU), src, b, bias)
+            _check(dev.gemm(a, w, bias=bias, epilogue=EPI_RELU), src, b, bias, 5)
 
 
 # 16x16 blocks (at most 256 of them): one row, row and column edges, K tails,
@@ -154,6 +214,7 @@ def test_fp32_pipeline_past_k_512(m, n, k):
     row-major B give the same bits."""
     note(f"fp32 pipeline {m}x{n}x{k}")
     device()
+    assert _tile(1, m, n, k) == 6
     a, b = _operands(1, m, n, k, 0, m + n + k)
     bias = torch.randn(n, device="cuda")
     got = dev.gemm(a, b, bias=bias, epilogue=EPI_RELU)
