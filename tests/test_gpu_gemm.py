@@ -76,38 +76,35 @@ def test_layout_matmul_packed(m, n, k):
     assert_gemm_close(to_host(got), ref, gemm_bound(a, w))
 
 
-# Packed B with N % 32 == 0 runs the LDS-DMA pipelined kernel: each of its
-# tile configurations (256x128, 128x128, 128x64 in 4 or 3 stages, 64x64,
-# chosen from the tile area the busiest CU computes, and K; 64x32 is covered
-# by test_packed_mid_batches), partial M and N tiles, a K tail with and
-# without full k-blocks, padded lda, addend and sigmoid; A rows that are not 16-byte
-# aligned (lda % 4 != 0) take the 4-byte DMA variant.
+# Packed B with N % 32 == 0: partial M and N tiles, a K tail with and without
+# full k-blocks, few and many k-blocks, rows of A of any pitch and alignment,
+# bias and addend, ReLU and sigmoid.  (Which tile runs each shape is decided by
+# the GEMM's time model; the split GEMM's own tests name the tiles.)
 PIPE_CASES = [
-    (4096, 1024, 845, 845, "128x128 tiles, unaligned A rows (4-byte DMA)"),
-    (4096, 512, 1023, 1023, "128x64 tiles, unaligned A rows"),
-    (4096, 256, 510, 510, "64x64 split-K tiles, unaligned A rows"),
+    (4096, 1024, 845, 845, "unaligned A rows, K tail"),
+    (4096, 512, 1023, 1023, "unaligned A rows"),
+    (4096, 256, 510, 510, "8-byte aligned A rows, K tail"),
     (1000, 96, 845, 845, "partial tiles and K tail, unaligned A rows"),
     (130, 64, 96, 97, "3 k-blocks, lda % 4 == 1"),
-    (4096, 1024, 864, 864, "128x128 tiles"),
-    (4096, 512, 1024, 1024, "128x64 tiles"),
-    (4096, 256, 512, 516, "64x64 tiles, padded lda"),
+    (4096, 1024, 864, 864, "whole tiles, 27 k-blocks"),
+    (4096, 512, 1024, 1024, "whole tiles, 32 k-blocks"),
+    (4096, 256, 512, 516, "padded lda"),
     (1000, 96, 845, 848, "partial M tile, partial N tile, K tail after 26 k-blocks"),
     (65, 32, 31, 32, "K < 32: tail only"),
     (33, 160, 64, 64, "2 k-blocks"),
-    (130, 64, 96, 100, "3 k-blocks (one full pipeline round), lda not a multiple of 32"),
+    (130, 64, 96, 100, "3 k-blocks, lda not a multiple of 32"),
     (7, 64, 300, 300, "tiny M"),
-    # few k-blocks in each tile class: the prologue and the mid-stage waits
-    # of the 4- and 3-stage pipelines
-    (4096, 1024, 40, 40, "128x64 tiles, two per CU (3 stages), 1 k-block + tail"),
-    (4096, 1024, 97, 97, "128x64 3-stage tiles, unaligned A, 3 k-blocks + tail"),
-    (4096, 1024, 128, 128, "128x64 3-stage tiles, 4 k-blocks"),
-    (4096, 1024, 544, 544, "128x128 tiles (K > 512), 17 k-blocks"),
-    (4096, 512, 160, 160, "128x64 tiles, 5 k-blocks"),
-    (4096, 512, 64, 67, "128x64 tiles, 2 k-blocks, unaligned A"),
-    (4096, 256, 224, 224, "64x64 split-K tiles, 7 k-blocks"),
-    (8192, 1024, 845, 845, "256x128 tiles, unaligned A rows (4-byte DMA), K tail"),
-    (8192, 1024, 1024, 1028, "256x128 tiles, padded lda"),
-    (8192, 1024, 544, 544, "256x128 tiles, 17 k-blocks"),
+    # few k-blocks: the pipelines' prologues
+    (4096, 1024, 40, 40, "1 k-block + tail"),
+    (4096, 1024, 97, 97, "unaligned A, 3 k-blocks + tail"),
+    (4096, 1024, 128, 128, "4 k-blocks"),
+    (4096, 1024, 544, 544, "17 k-blocks"),
+    (4096, 512, 160, 160, "5 k-blocks"),
+    (4096, 512, 64, 67, "2 k-blocks, unaligned A"),
+    (4096, 256, 224, 224, "7 k-blocks"),
+    (8192, 1024, 845, 845, "unaligned A rows, K tail, several rounds"),
+    (8192, 1024, 1024, 1028, "padded lda, several rounds"),
+    (8192, 1024, 544, 544, "17 k-blocks, several rounds"),
 ]
 
 
@@ -385,12 +382,15 @@ def test_small_batch_tower_graph_replays(batch_rows):
         torch.cuda.synchronize()
 
 
-@pytest.mark.parametrize("m,n,k,ldb_pad", [(1, 1024, 4096, 0), (4096, 512, 256, 1)])
+@pytest.mark.parametrize("m,n,k,ldb_pad", [(1, 1024, 4096, 0), (64, 500, 4096, 1),
+                                           (217, 448, 2048, 0), (128, 1000, 3100, 1),
+                                           (4096, 512, 256, 1)])
 def test_gemm_captured_without_warm_up(m, n, k, ldb_pad):
-    """GEMMs that use the per-stream workspace (a K-split small product, a
-    row-major B with unaligned rows) captured on a fresh stream with no call
-    before: no allocation happens under capture (the library takes a path
-    without workspace), and the replays give the oracle's result."""
+    """GEMMs that split K over workgroups, and so use the per-stream workspace
+    (16x16 and 32x32 blocks, packed and unaligned row-major B; the last shape
+    uses none), captured on a fresh stream with no call before: no allocation
+    happens under capture (the library takes a path without workspace), and
+    the replays give the oracle's result."""
     note(f"GEMM captured without warm-up {m}x{n}x{k} ldb+{ldb_pad}")
     g = workloads.rng(m + n + k)
     a = g.standard_normal((m, k)).astype(np.float32)
@@ -412,42 +412,44 @@ def test_gemm_captured_without_warm_up(m, n, k, ldb_pad):
         assert_gemm_close(to_host(out), ref, gemm_bound(a, w, np.broadcast_to(bias, ref.shape)))
 
 
-def test_graph_replays_after_the_workspace_grows():
-    """A GEMM that packs unaligned B rows into the workspace, captured after a
-    warm-up on the capture stream; eager calls of the same thread on that
-    stream then need a larger workspace (it grows; the outgrown one, which
-    the graph holds, is kept): later replays equal the first bit for bit and
-    stay within the GEMM bound."""
-    note("graph replay after the workspace grows")
+@pytest.mark.parametrize("m,n,k", [(1, 1024, 4096), (217, 448, 2048)])
+def test_graph_replays_after_the_workspace_grows(m, n, k):
+    """A GEMM that splits K over workgroups, its partial sums (16 KiB, 760 KiB)
+    in the stream's first workspace of 1 MiB, captured after a warm-up on the
+    capture stream.  Eager calls of the same thread on that stream then need
+    more (a hash table of 2^20 slots and the keys' numbers: it grows; the
+    outgrown one, which the graph holds, is kept), and torch's allocations
+    would take the place of one given back: later replays equal the first bit
+    for bit and stay within the GEMM bound."""
+    note(f"graph replay after the workspace grows {m}x{n}x{k}")
     g = workloads.rng(77)
-    m, n, k = 600, 1024, 512
     a = g.standard_normal((m, k)).astype(np.float32)
-    wide = (g.standard_normal((k, n + 1)) / np.sqrt(k)).astype(np.float32)
-    w = np.ascontiguousarray(wide[:, :n])
+    w = (g.standard_normal((k, n)) / np.sqrt(k)).astype(np.float32)
     bias = (g.standard_normal(n) * 0.1).astype(np.float32)
-    da, db, dbias = to_dev(a), to_dev(wide)[:, :n], to_dev(bias)
+    da, db, dbias = to_dev(a), to_dev(w), to_dev(bias)
     out = torch.empty((m, n), dtype=torch.float32, device=device())
     graph = CapturedGraph(lambda: dev.gemm(da, db, bias=dbias, epilogue=EPI_RELU, out=out))
     first = to_host(graph.replay()).copy()
     ref = ora.dense_layer(a, w, bias, 1)
     assert_gemm_close(first, ref, gemm_bound(a, w, np.broadcast_to(bias, ref.shape)))
-    big_k = 4096
-    a2 = g.standard_normal((m, big_k)).astype(np.float32)
-    wide2 = (g.standard_normal((big_k, 2 * n + 1)) / np.sqrt(big_k)).astype(np.float32)
+    keys = to_dev(g.integers(0, 300_000, size=400_000).astype(np.int64))
+    table = torch.zeros((300_000, 4), device=device())
     with torch.cuda.stream(graph.stream):
-        big = dev.gemm(to_dev(a2), to_dev(wide2)[:, :2 * n])
+        uniq, index, _ = dev.unique_gather(table, keys)
     torch.cuda.synchronize()
-    assert_gemm_close(to_host(big), ora.matmul(a2, np.ascontiguousarray(wide2[:, :2 * n])),
-                      gemm_bound(a2, wide2[:, :2 * n]))
+    assert torch.equal(uniq[index.long()], keys)
+    filled = [torch.full((1 << 18,), float(i), device=device()) for i in range(64)]
     for _ in range(3):
         out.zero_()
         np.testing.assert_array_equal(to_host(graph.replay()), first)
+    for i, f in enumerate(filled):
+        assert (f == i).all()
 
 
 def test_workspace_calls_from_two_threads_on_one_stream():
-    """Two threads enqueue workspace-using calls (per-call packing of
-    unaligned B rows, K split, the any-order segment reduction) on one stream
-    at once, each in its own order, so their launches interleave and each
+    """Two threads enqueue workspace-using calls (K split over workgroups in
+    16x16 and 32x32 blocks, the any-order segment reduction) on one stream at
+    once, each in its own order, so their launches interleave and each
     thread's workspace grows meanwhile: every result equals the same call's
     single-threaded result bit for bit."""
     import threading
@@ -455,8 +457,8 @@ def test_workspace_calls_from_two_threads_on_one_stream():
     g = workloads.rng(78)
     stream = torch.cuda.Stream()
     calls = []
-    for m, n, k, pad in [(600, 2048, 1024, 1), (1, 1024, 4096, 0), (300, 1000, 2100, 3),
-                         (64, 512, 4096, 0), (600, 2048, 2048, 1)]:
+    for m, n, k, pad in [(217, 448, 2048, 1), (1, 1024, 4096, 0), (128, 1000, 3100, 3),
+                         (64, 512, 4096, 0), (100, 1024, 4096, 1)]:
         a = to_dev(g.standard_normal((m, k)).astype(np.float32))
         b = to_dev((g.standard_normal((k, n + pad)) / np.sqrt(k)).astype(np.float32))[:, :n]
         calls.append(lambda a=a, b=b: dev.gemm(a, b, epilogue=EPI_RELU))
@@ -647,13 +649,7 @@ def test_batch_matmul_add_sigmoid_broadcasts(bias_shape, rhs_batched):
     np.testing.assert_allclose(got, ref, rtol=0, atol=1e-5)
 
 
-# (each shape has n % 32 == 0 and at least 128 64x64 tiles, the condition for
-# the pipelined kernel.  Rows of B that are 16-byte aligned (n + ldb_pad a
-# multiple of 4) are read in place; the others need m >= 512 and are packed
-# per call, the packer grouping 1, 2 or 4 n-panels per workgroup by grid size:
-# (1, 8192, 64, 33, 7) takes 1 and (70, 512, 224, 64, 3) 2 with a remainder
-# group.  The tile rule gives 64x64, 128x64 in 4 and 3 stages, and a grid of
-# 1.25 CU rounds among these shapes.)
+# (n % 32 == 0; rows of B of any pitch and alignment are read in place)
 @pytest.mark.parametrize("batch,m,n,k,ldb_pad", [(1, 2048, 320, 845, 80), (1, 4096, 512, 1024, 0),
                                                  (3, 1024, 256, 200, 0), (1, 8192, 64, 33, 7),
                                                  (2, 4000, 96, 64, 32), (32, 512, 256, 256, 0),
@@ -662,15 +658,13 @@ def test_batch_matmul_add_sigmoid_broadcasts(bias_shape, rhs_batched):
                                                  (2, 4096, 1024, 1024, 0), (1, 8192, 1024, 845, 3),
                                                  (3, 40, 64, 96, 0), (4, 33, 96, 845, 5),
                                                  (1, 500, 2048, 1024, 1), (2, 256, 2048, 512, 3)])
-def test_row_major_b_packed_per_call(batch, m, n, k, ldb_pad):
-    """Large row-major-B GEMMs run the pipelined kernel, on B read in place or
-    packed into the stream workspace: within tolerance of OpenBLAS, and
-    bit-identical to the same GEMM on weights packed ahead of time (so the
-    in-place reads and the per-call packing both equal the layout_matmul
-    packer, K tails and strided B included, and the pipelined kernel ran).
+def test_row_major_b_read_in_place(batch, m, n, k, ldb_pad):
+    """Row-major-B GEMMs of more than one round of 32x32 blocks read B in
+    place: within tolerance of OpenBLAS, and bit-identical to the same GEMM on
+    weights packed ahead of time, K tails and strided B included.
     Batches of at most 256 32x32 blocks run the small kernel on both forms
     (batched packed B included), bit-identical likewise."""
-    note(f"row-major B packed per call b={batch} {m}x{n}x{k} ldb+{ldb_pad}")
+    note(f"row-major B in place b={batch} {m}x{n}x{k} ldb+{ldb_pad}")
     g = workloads.rng(m + n + k + batch)
     a = g.standard_normal((batch, m, k)).astype(np.float32)
     wide = (g.standard_normal((batch, k, n + ldb_pad)) * 0.05).astype(np.float32)
@@ -731,8 +725,7 @@ def test_packed_small_batches(batch, m, n, k):
                                         (4000, 288, 845, 3)])
 def test_packed_mid_batches(m, n, k, col0):
     """Batches between one round of 32x32 blocks and two rounds of 64x64
-    tiles run 64x32 tiles of the pipelined kernel (16- and 4-byte A DMAs, K
-    tails): within the GEMM bound of OpenBLAS, and bit-identical to the same
+    tiles (A rows of any alignment, K tails): within the GEMM bound of OpenBLAS, and bit-identical to the same
     GEMM on row-major B."""
     note(f"packed mid batch {m}x{n}x{k} col0={col0}")
     g = workloads.rng(5 * m + n + k + col0)
@@ -748,33 +741,30 @@ def test_packed_mid_batches(m, n, k, col0):
     np.testing.assert_array_equal(got, rm)
 
 
-# N % 32 != 0 with more than one round of 32x32 blocks in the full panels:
-# the pipelined kernel with a partial last panel (packed B, and row-major B
-# with 16-byte aligned rows read in place; other row-major B is packed per
-# call, tail columns included, and runs as packed B), or, where the extra
-# column of tiles costs a CU round, the full panels and then the tail
-# columns through the small kernel (N % 32 > 4) or the GEMV kernel.
+# N % 32 != 0 with more than one round of 32x32 blocks in the full panels: one
+# launch with a partial last panel, or the full panels and then the tail columns
+# through the small kernel (N % 32 > 4) or the GEMV kernel, as the time model
+# decides; B packed or row-major, rows of any alignment.
 N_TAIL_CASES = [
     (1, 4096, 1000, 1024, "8 tail columns"),
-    (1, 4096, 515, 845, "3 tail columns; row-major rows unaligned (packed per call), K tail"),
+    (1, 4096, 515, 845, "3 tail columns; row-major rows unaligned, K tail"),
     (1, 2048, 300, 845, "12 tail columns, K tail"),
     (3, 1024, 100, 64, "batched, 4 tail columns"),
-    (1, 8200, 33, 256, "one full panel, 1 tail column (row-major: packed per call)"),
+    (1, 8200, 33, 256, "one full panel, 1 tail column"),
     (2, 777, 620, 100, "batched, partial M tile, 12 tail columns, K tail"),
-    (1, 4096, 1001, 40, "unaligned rows (packed per call), 1 k-block + K tail"),
-    (1, 8192, 1000, 864, "256x128 tiles with a partial panel"),
-    (1, 1200, 340, 512, "64x32 tiles with a partial panel"),
+    (1, 4096, 1001, 40, "unaligned rows, 1 k-block + K tail"),
+    (1, 8192, 1000, 864, "8 tail columns, several rounds"),
+    (1, 1200, 340, 512, "20 tail columns, one round"),
     (1, 4096, 1000, 20, "K < 32 (K tail only), partial panel"),
-    (1, 4096, 521, 1024, "unaligned rows, two launches (a fifth round of tiles)"),
-    (2, 2048, 1001, 97, "batched, unaligned rows: K*N odd, batch strides of the per-call pack aligned"),
+    (1, 4096, 521, 1024, "unaligned rows, 9 tail columns"),
+    (2, 2048, 1001, 97, "batched, unaligned rows: K*N odd"),
 ]
 
 
 @pytest.mark.parametrize("batch,m,n,k,what", N_TAIL_CASES)
 def test_n_tail_split(batch, m, n, k, what):
     """Within the GEMM bound of OpenBLAS with bias and ReLU, and with an
-    addend and sigmoid; packed B and row-major B (read in place, or packed
-    per call) bit-identical."""
+    addend and sigmoid; packed B and row-major B bit-identical."""
     note(f"N-tail split b={batch} {m}x{n}x{k}: {what}")
     g = workloads.rng(3 * m + n + k + batch)
     a = g.standard_normal((batch, m, k)).astype(np.float32)
@@ -801,8 +791,8 @@ def test_n_tail_split(batch, m, n, k, what):
             assert_gemm_close(got_b[z], ref, gemm_bound(a[z], w[z], np.broadcast_to(bias, ref.shape)))
 
 
-# 4 < N < 32 with more than one round of 32x32 blocks: 64x32 pipelined tiles
-# with one partial panel and no full ones (B by 4-byte DMAs from any ldb);
+# 4 < N < 32 with more than one round of 32x32 blocks: tiles with one partial
+# panel and no full ones;
 # also the tail columns of a two-launch GEMM at such M
 SKINNY_PIPE_CASES = [
     (1, 16384, 16, 1024, 0, 0, "one round of 64x32 tiles"),
@@ -810,7 +800,7 @@ SKINNY_PIPE_CASES = [
     (1, 65536, 8, 256, 0, 0, "1024 tiles: several rounds of three a CU"),
     (1, 20000, 31, 100, 0, 0, "partial M tile, K tail"),
     (1, 12000, 7, 300, 0, 0, "ldb = 7 (rows not 16-byte aligned)"),
-    (1, 10000, 12, 96, 3, 1, "ldb padded, A from a column offset (4-byte A DMAs)"),
+    (1, 10000, 12, 96, 3, 1, "ldb padded, A from a column offset (4-byte aligned)"),
     (3, 4000, 12, 64, 0, 0, "batched: 375 blocks over the batch"),
     (1, 9000, 5, 40, 0, 0, "N = 5, one k-block and a K tail"),
     (1, 16384, 1009, 64, 1, 0, "row-major, unaligned rows: pipelined full panels, tail of 17 columns pipelined"),
@@ -908,8 +898,7 @@ def test_k_zero_is_the_epilogue_alone(m, n):
 @pytest.mark.parametrize("m,n,k,col0", [(2048, 512, 256, 1), (8192, 64, 333, 3)])
 def test_pipeline_misaligned_a_base(m, n, k, col0):
     """A starting mid-row of a wider buffer (base not 16-byte aligned, lda a
-    multiple of 4): the 4-byte DMA variant, bit-identical between packed and
-    per-call-packed row-major B."""
+    multiple of 4), bit-identical between packed and row-major B."""
     note(f"misaligned A base {m}x{n}x{k} col0={col0}")
     g = workloads.rng(m + n + k + col0)
     buf = g.standard_normal((m, k + 8)).astype(np.float32)
@@ -930,7 +919,7 @@ def _sweep_case(seed):
     """A seeded random GEMM call: shape, batch, B layout, operand strides and
     epilogue drawn so that every dispatch path turns up over the seeds (GEMV,
     small kernel with and without K split, 64x32, 128x64, 128x128 and
-    256x128 tiles, partial panels, N < 32, K tails, per-call packing)."""
+    256x128 tiles, partial panels, N < 32, K tails, row-major and packed B)."""
     g = workloads.rng(1000 + seed)
     batch = int(g.choice([1, 1, 1, 2, 3]))
     m = _log_uniform(g, 1, 9000) if g.random() < 0.5 else _log_uniform(g, 512, 9000)
@@ -1000,10 +989,9 @@ def test_gemm_random_shapes(seed):
 def test_custom_calls_from_concurrent_threads():
     """The synchronous custom calls run on a stream of the calling thread:
     threads calling __matmul_add_relu at once (host buffers staged through
-    each thread's scratch; threads 2 and 3 have at least 128 64x64 tiles and
-    run the pipelined kernel) each get their own result; so do their device
-    calls on their own streams, where threads 2 and 3 pack an unaligned
-    row-major B into that stream's workspace."""
+    each thread's scratch) each get their own result; so do their device
+    calls on their own streams, on unaligned row-major B and with K split over
+    workgroups in that stream's workspace."""
     import threading
     note("custom calls from 4 threads")
     g = workloads.rng(77)
@@ -1022,11 +1010,14 @@ def test_custom_calls_from_concurrent_threads():
             ref = ora.matmul_add_relu(e, a, b)
             bound = gemm_bound(a, b, e)
             k, n = b.shape
+            a2, b2 = np.resize(a, (1 + k // 8 % 4, 4096)), np.resize(b, (4096, 512))
+            ref2, bound2 = ora.matmul(a2, b2), gemm_bound(a2, b2)
             wide = np.zeros((k, n + 3), np.float32)  # rows not 16-byte aligned
             wide[:, :n] = b
             s = torch.cuda.Stream(device=device())
             with torch.cuda.stream(s):
                 da, de, db = to_dev(a), to_dev(e), to_dev(wide)[:, :n]
+                da2, db2 = to_dev(a2), to_dev(b2)
                 s.synchronize()
                 for _ in range(5):
                     xla.matmul_add_relu(z, e, a, b, out)
@@ -1034,6 +1025,9 @@ def test_custom_calls_from_concurrent_threads():
                     got = dev.gemm(da, db, addend=de, epilogue=EPI_RELU)
                     s.synchronize()
                     assert_gemm_close(to_host(got), ref, bound)
+                    got = dev.gemm(da2, db2)
+                    s.synchronize()
+                    assert_gemm_close(to_host(got), ref2, bound2)
         except Exception as ex:  # reported below
             errors.append(ex)
 
