@@ -177,6 +177,18 @@ def test_row_stride_past_32_bit_offsets():
             _check(dev.gemm(a, w, bias=bias, epilogue=EPI_RELU), src, b, bias, 5)
 
 
+def test_b_row_stride_past_32_bit_offsets():
+    """Row-major B with rows 2^27 floats apart: the tile kernel."""
+    note("GEMM with a row stride of B of 2^27 floats")
+    device()
+    m, n, k, ldb = 300, 1000, 4, 1 << 27
+    a, src = _operands(1, m, n, k, 0, 4)
+    b = torch.empty((k - 1) * ldb + n, device="cuda").as_strided((k, n), (ldb, 1))
+    b.copy_(src)
+    bias = torch.randn(n, device="cuda")
+    _check(dev.gemm(a, b, bias=bias, epilogue=EPI_RELU), a, src, bias, 5)
+
+
 # 16x16 blocks (at most 256 of them): one row, row and column edges, K tails,
 # K < 32, partial panels of 1-31 columns, K split over workgroups (K >= 2048)
 TINY_CASES = [(1, 1, 512, 1024), (1, 17, 33, 64), (1, 16, 47, 545), (1, 15, 8, 20), (1, 256, 256, 31),
