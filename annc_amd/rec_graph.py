@@ -97,12 +97,12 @@ class MLPTower:
         hidden-layer weight: up to 4096 rows are one round of workgroups, and
         each further round streams the weight again, while the GEMM's tiles
         follow the batch.  Steps of towers with a tail of K -> N -> 1, fused /
-        unfused, us: 512 -> 256 at 4096 rows 45.0 / 48.2, 4112 63.9 / 62.1, 5120
-        64.5 / 62.6, 8192 75.2 / 74.5, 16384 134 / 127; 1024 -> 256 4112 104 / 94,
-        16384 259 / 234; 1024 -> 128 5120 65.1 / 62.2; smaller weights 256 -> 128
-        5120 26.7 / 29.9, 16384 45.6 / 49.1; 512 -> 128 5120 42.1 / 44.4, 16384
-        72.9 / 73.0, 32768 137 / 131; 512 -> 64 32768 119 / 122; 256 -> 256 16384
-        55.4 / 56.9, 32768 97 / 86."""
+        unfused, us: 512 -> 256 at 4096 rows 44.9 / 47.9, 4112 63.4 / 61.2, 5120
+        64.1 / 61.7, 8192 74.3 / 73.5, 16384 129 / 124; 1024 -> 256 4112 78 / 69,
+        16384 171 / 150; 1024 -> 128 5120 65.7 / 63.8; smaller weights 256 -> 128
+        5120 26.8 / 29.9, 16384 46.0 / 50.1; 512 -> 128 5120 42.0 / 44.1, 16384
+        74.2 / 73.7, 32768 138 / 132; 512 -> 64 32768 119 / 122; 256 -> 256 16384
+        56.1 / 56.3, 32768 97 / 87."""
         if not self.fused_tail or rows < self.fuse_min_rows:
             return False
         hid = self.layers[-2].weight

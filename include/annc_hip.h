@@ -191,7 +191,12 @@ int annc_hip_layout_matmul_pack_rhs(void* stream, int64_t k, int64_t n, const fl
 
 /* ------------------------------------------------------------------------ */
 /* Device GEMM (engine behind __matmul* / __batch_matmul / __layout_matmul)  */
-/*   C[z] = epi( A[z] . B[z] (+ E[z]) (+ bias) )   row-major, fp32 MFMA       */
+/*   C[z] = epi( A[z] . B[z] (+ E[z]) (+ bias) )   row-major, fp32            */
+/* Products run on the fp32 matrix instruction or, large ones, as six bf16   */
+/* products of the operands' three pieces with fp32 accumulation: closer to  */
+/* the 64-bit result on dense operands, within 2^-23 of a single product     */
+/* (the fp32 instruction: 2^-24), and with its results for infinite, NaN and */
+/* denormal operands.                                                         */
 /* b_packed = 1: B is in annc_layout_matmul_pack_rhs order (ldb ignored).    */
 /* epilogue bits: ANNC_EPI_RELU = max(x, 0) as std::max(x, 0.f)              */
 /* (gemm_rewriter.cc:278-280); ANNC_EPI_SIGMOID = 1/(1+exp(-x)).             */
